@@ -916,6 +916,39 @@ def test_shadow_forward_positions_and_flags(cufk, device, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,N", [(1500, 384), (2049, 384), (1500, 697), (2049, 697), (900, 1020), (2049, 1020),
+                                 (700, 1500), (700, 2049)])
+def test_half_positions_are_the_float_positions_rounded_once(cufk, device, dtype, B, N):
+    """Every forward plan of more than 256 steps, over 1.7 to 6.3 million coordinates each: the kept
+    float positions round to the stored output, which the plain and the fused forwards store bit for
+    bit alike.  A conversion fused into the placing multiply-add rounds the exact sum instead, which
+    differs where the float position is a tie between two float16 (one coordinate in about 10^4)."""
+    lib = _abi_fused()
+    gen = torch.Generator(device=device).manual_seed(B + N)
+    normal = lambda *s: torch.randn(*s, generator=gen, device=device)  # noqa: E731
+    L = (0.145 + 0.01 * normal(B, N - 1)).to(dtype)
+    A = (2.05 + 0.08 * normal(B, N - 2)).to(dtype)
+    D = (2.0 * normal(B, N - 3)).to(dtype)
+    an = _anchors3(_inputs(1, 8, seed=N, anchors=True, dtype=dtype), dtype, device)
+    xyz, pos, _ = _shadow_forward(lib, L, A, D, an)
+    assert torch.equal(pos.to(dtype), xyz)
+    plain, reg = _flagged_forward(lib, L, A, D, an)
+    assert torch.equal(plain, xyz)
+    p = lambda t: t.data_ptr()  # noqa: E731
+    st = torch.cuda.current_stream().cuda_stream
+    target = (pos + 0.3 * normal(B, N, 3)).to(dtype)
+    loss, rec = torch.empty(B, device=device, dtype=dtype), torch.empty(B, 24, device=device, dtype=torch.float64)
+    fused = torch.empty_like(xyz)
+    assert lib.cufk_reconstruct_loss_fwd(_CODES[dtype], p(L), p(A), p(D), *map(p, an), p(target), p(fused), p(reg),
+                                         p(loss), B, N, st) == 0
+    assert torch.equal(fused, xyz)
+    fused.zero_()
+    assert lib.cufk_reconstruct_superposed_fwd(_CODES[dtype], 1, p(L), p(A), p(D), *map(p, an), p(target), p(fused),
+                                               p(reg), p(loss), p(rec), B, N, st) == 0
+    assert torch.equal(fused, xyz)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("N", [4, 5, 70, 259, 1028, 2049, 2051])
 def test_shadow_backward_is_the_float32_adjoint(cufk, device, dtype, N):
     """Over the kept float positions the half-type backward runs the float32 position-based
