@@ -95,6 +95,24 @@ def test_table_sin_cos_accuracy_and_norm(wide, bar):
     assert np.abs(s * s + co * co - 1.0).max() <= 2e-12
 
 
+def test_huge_angles_polynomials():
+    """The checked form's Taylor polynomials over the whole remainder range, in extended precision with
+    the coefficients parsed from the source: what they leave out is far below a double's rounding."""
+    text = SRC.read_text()
+    body = text[text.index("void sin_cos_tab(float xf"):]
+    body = body[: body.index("\n}\n")]
+    sine = re.search(r"sr = fma\(r \* u, fma\(u, fma\(u, (-?)1.0 / ([\d.]+), 1.0 / ([\d.]+)\), -1.0 / ([\d.]+)\), r\);", body)
+    cosine = re.search(r"w = u \* fma\(u, fma\(u, (-?)1.0 / ([\d.]+), 1.0 / ([\d.]+)\), (-0.5)\);", body)
+    ld = np.longdouble
+    s7, s5, s3 = (ld(1) / ld(v) for v in sine.groups()[1:])
+    c6, c4 = (ld(1) / ld(v) for v in cosine.groups()[1:3])
+    assert sine.group(1) == cosine.group(1) == "-"
+    r = np.linspace(-np.pi / 128, np.pi / 128, 20001).astype(ld)
+    u = r * r
+    assert np.abs(r + r * u * (u * (u * -s7 + s5) - s3) - np.sin(r)).max() <= 1e-19
+    assert np.abs(u * (u * (u * -c6 + c4) - ld(0.5)) - (np.cos(r) - 1)).max() <= 1e-17
+
+
 def test_taylor_cubic_would_fail_the_bar():
     k_round, inv_step, step, _s1, c2, table = _constants()
     x = _angles()
