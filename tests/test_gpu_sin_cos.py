@@ -41,7 +41,7 @@ def _forward(device, batch, points, lengths, first_angle, angle, dihedral):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("batch,points", SHAPES)
-@pytest.mark.parametrize("huge", [True])
+@pytest.mark.parametrize("huge", [True, False])
 def test_first_angle(device, batch, points, huge):
     """x2 = (-cos, sin, 0) of the first angle for bonds (0, 1)."""
     a = _angles(batch, huge, 1)
