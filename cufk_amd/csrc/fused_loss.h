@@ -91,11 +91,18 @@ __device__ __forceinline__ auto make_residual(R w, const double* __restrict__ re
 // noise (MSD 3e-6 nm^2), 2e-9 nm^2, 7e-4 relative; the RMSD and the scale of its gradient,
 // 1 / (2 rmsd), carry half that relative error (2.5e-4 measured).  Chains fitted more closely
 // than that have a relatively coarser loss.
-template <int LossKind, typename R> struct LossAccumulator {
+//
+// S2 is the type of those products and squares: R, or double in the forward plans of one or two waves
+// with eight or twelve steps per thread.  Such a chain had at least half as many steps per thread in the
+// staged forward, and the floor above grows with the extent of a thread's points squared: at 3000 x 700
+// with 1e-3 nm of noise the loss was 2.6e-4 off (rms, relative) with eight float steps per thread, 6.8e-4
+// with twelve, and is 1.1e-7 off with twelve in double, for no time (28.5 us for the forward either way,
+// MI355X).
+template <int LossKind, typename R, typename S2 = R> struct LossAccumulator {
   static constexpr bool kSuperposed = LossKind == kLossSuperposed;
   double acc = 0.0;
   double s1[kSuperposed ? 6 : 1] = {};   // sum a, sum b (about xl, tl)
-  R s2[kSuperposed ? 11 : 1] = {};       // sum a b^T (row-major), sum |a|^2, sum |b|^2
+  S2 s2[kSuperposed ? 11 : 1] = {};      // sum a b^T (row-major), sum |a|^2, sum |b|^2
   int m = 0;                             // points summed by this thread
   V3<R> cx = {R(0), R(0), R(0)}, ct = {R(0), R(0), R(0)};  // the chain's shift points
   V3<R> xl = {R(0), R(0), R(0)}, tl = {R(0), R(0), R(0)};  // this thread's
@@ -114,7 +121,7 @@ template <int LossKind, typename R> struct LossAccumulator {
   __device__ __forceinline__ void add(V3<R> xs, V3<R> t) {
     if constexpr (kSuperposed) {
       const V3<R> av = xs - xl, bv = t - tl;
-      const R a[3] = {av.x, av.y, av.z}, b[3] = {bv.x, bv.y, bv.z};
+      const S2 a[3] = {av.x, av.y, av.z}, b[3] = {bv.x, bv.y, bv.z};
 #pragma unroll
       for (int i = 0; i < 3; ++i) {
         s1[i] += static_cast<double>(a[i]);

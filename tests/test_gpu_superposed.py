@@ -159,6 +159,25 @@ def test_rmsd_fp32_small_deviation(cufk, device, squared):
     assert max(gerr) <= (5e-5 if squared else 1e-3)
 
 
+@pytest.mark.parametrize("B,N", [(2049, 300), (3000, 514), (2049, 700), (1100, 1000), (2049, 1000)])
+def test_rmsd_fp32_small_deviation_long_runs(cufk, device, B, N):
+    """The forward plans of eight and twelve steps per thread in one or two waves sum the products in
+    double: with 1e-3 nm of noise the loss is the superposition of the stored positions to 1e-5
+    relative (7e-7 measured: the rounding of differences within a thread's run of points, 1e-7 of about
+    1 nm against 1e-3 nm, averaged over the chain; float products were 2e-4 to 3e-3 off)."""
+    gen = torch.Generator(device=device).manual_seed(N)
+    normal = lambda *s: torch.randn(*s, generator=gen, device=device)  # noqa: E731
+    L, A, D = 0.145 + 0.01 * normal(B, N - 1), 2.05 + 0.08 * normal(B, N - 2), 2.0 * normal(B, N - 3)
+    stored = cufk.reconstruct(L, A, D)
+    target = stored + 1e-3 * normal(B, N, 3)
+    pick = torch.arange(0, B, B // 100, device=device)
+    got = cufk.reconstruct_rmsd(L, A, D, target)[pick].double().cpu().numpy()
+    want = o.superposed_loss(stored[pick].double().cpu().numpy(), target[pick].double().cpu().numpy(), squared=False)
+    err = np.abs(got / want - 1.0).max()
+    print(f"{B} x {N}: {err:.2e}")
+    assert err <= 1e-5
+
+
 def test_rmsd_matches_the_unfused_composition(cufk, device):
     """float64: the fused loss and gradients equal the unfused composition's within 1e-12 / 1e-10."""
     d = _case(4, 300, seed=21, dtype=torch.float64)
