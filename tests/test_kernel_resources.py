@@ -73,3 +73,9 @@ def test_double_forwards_of_four_steps_run_four_waves():
 def test_double_forwards_do_not_spill():
     for name, k in _named(r"\d(reconstruct(_\w+)?_forward|long_forward_segments)_kernelId").items():
         assert k[".vgpr_spill_count"] == 0 and k[".private_segment_fixed_size"] == 0, name
+
+
+def test_saved_backwards_do_not_spill():
+    """The exact path of a refused chain shares the registers of the position-based one."""
+    for name, k in _named(r"reconstruct(_loss)?_backward(_saved)?_kernelI(f|d|DF16)").items():
+        assert k[".vgpr_spill_count"] == 0 and k[".private_segment_fixed_size"] == 0, name
