@@ -38,7 +38,6 @@ template <> struct TileVec<8, 2> { typedef u32x2 Local; typedef u32x2a2 Global; 
 // (half types, N = 4 or 12).  A run's first vector sits at kStride vectors per lane, kStride odd:
 // 16 lanes reading one 16-byte vector each (32 reading 8 bytes) then cover all 64 banks once.
 template <typename T, int N> struct LaneTile {
-  static constexpr int kRun = N;
   static constexpr int kBytes = N * static_cast<int>(sizeof(T));
   static constexpr int kVecBytes = kBytes % 16 == 0 ? 16 : 8;
   static_assert(kBytes % kVecBytes == 0, "a lane's run is whole vectors");
@@ -101,7 +100,7 @@ __device__ __forceinline__ void pack_run(const R (&v)[N], Vec (&run)[NV]) {
 }
 
 // A window of one row on its way from HBM to the lanes' runs: elements [start, end) of the row (end
-// - start may be 64 kRun and more, or <= 0).  fetch() issues the loads, to_runs() hands every lane its
+// - start may be 64 runs and more, or <= 0).  fetch() issues the loads, to_runs() hands every lane its
 // run.  Every lane issues every load, those past the row's end at its last whole vector instead: with
 // no branch around them, what is loaded before the rows need not wait for the rows (with an exec mask
 // around each load the compiler waits for all of them at once: at B = 4096, N = 2049, whose last wave
@@ -138,7 +137,7 @@ template <typename T, typename Tile> struct WindowLoad {
     tail = row[at];
   }
 
-  // n = end - start; elements past them are `pad`.  `full` (uniform): n >= 64 kRun.
+  // n = end - start; elements past them are `pad`.  `full` (uniform): n holds 64 whole runs.
   __device__ __forceinline__ void to_runs(void* tile, Vec (&run)[NV], int n, bool full, T pad, int lane) const {
     Vec* const t = static_cast<Vec*>(tile);
     wave_lds_order();

@@ -10,7 +10,8 @@
 // One workgroup of W wave64s reconstructs one chain; lane t owns the K consecutive steps
 // [tK, tK+K) (blocked arrangement, as in the reference block.cu:187), runs them as a serial
 // scan in registers and only lane totals cross lanes (wave64 DPP scan, then an LDS carry across
-// waves).  Rows move between HBM and LDS as coalesced 16-byte streams.
+// waves).  Rows move between HBM and a wave's registers through a wave-private LDS tile (lane_tile.h);
+// the recompute backward and the long chains' backward stage whole rows in LDS (staging.h).
 #include "launch.h"
 
 #include <hip/hip_runtime.h>
@@ -58,24 +59,22 @@ namespace cufk_amd {
 
 // ---------------------------------------------------------------------------- plans
 
-// (waves W, items per lane K), capacity 64*W*K steps; the smallest plan holding the chain.
-// Eight items per lane measured fastest at N = 2049 for both the forward and the
-// position-based backward (K = 16 runs out of registers and waves, K = 4 pays the lane scan
-// on too few items).  The exact backward uses the same plans.  The kernels stage rows with one
-// word of padding per lane: at (4, 8) that lets five forward workgroups (three backward)
-// share a CU instead of four (two).
+// (waves W, items per lane K), capacity 64*W*K steps; the smallest plan holding the chain.  The
+// backwards take these plans, and the forwards where with_forward_plan has none of its own.
+// Eight items per lane measured fastest at N = 2049 (K = 16 runs out of registers and waves, K = 4
+// pays the lane scan on too few items).  The exact backward uses the same plans.
 //
 // Small grids (`groups` workgroups of one chain each, at most kLatencyWaves waves under the
 // eight-item plan, four per SIMD) run latency-bound: a lone wave per SIMD waits on every
 // dependent instruction.  There the chain takes twice the waves with four items per lane,
-// halving each lane's serial scan.  Measured on MI355X (forward + position-based backward,
-// back-to-back launches): B=1024, N=384: 13.6 against 15.1 us; B=512, N=384: 11.4 against
-// 12.5 us; B=2048, N=700: 30.1 against 33.2 us.
-constexpr int kScanPad = 1;
+// halving each lane's serial scan.  Measured on MI355X (forward + position-based backward in a graph,
+// against eight items): 512 x 384 11.0 against 11.4 us, 1024 x 384 13.4 against 13.9, float64 1024 x 384
+// 19.9 against 22.0, 2048 x 1026 61.4 against 62.5.  Float32 at the upper end would take eight since its
+// rows are in registers: 4096 x 384 28.4 against 26.5, 2048 x 700 26.5 against 25.2.
 constexpr int64_t kLatencyWaves = 4096;
 //
 // Every plan gives each of its waves some of the chain's steps (a wave past the chain would still
-// run the lane scan, lane_scan_chain): where four waves of four or eight steps would leave the
+// run the scan): where four waves of four or eight steps would leave the
 // last one idle (513-768 and 1025-1536 steps), the chain takes three.
 template <typename Fn> int with_scan_plan(int64_t groups, int steps, Fn&& fn) {
   if (steps <= 256) return fn.template operator()<1, 4>();
@@ -107,7 +106,7 @@ template <typename Fn> int with_scan_plan(int64_t groups, int steps, Fn&& fn) {
 // (1, 16) at 769-1024 steps and (2, 12) at 1025-1536 gain another 1-3 % for plain forwards and lose
 // 6-40 % for the fused losses, whose targets need as many registers again.  Double chains keep the
 // general plans: at twelve steps per lane they would not fit the registers.
-constexpr int64_t kSplitGroups = 2048;  // chains up to which twice the waves per chain pay
+constexpr int64_t kSplitGroups = 2048;  // chains up to which two or three waves per chain pay, not one
 template <typename T, typename Fn> int with_forward_plan(int64_t groups, int steps, int chain_steps, Fn&& fn) {
   if (chain_steps < tiny_steps<T>()) return fn.template operator()<1, 4, true>();
   if constexpr (sizeof(T) < 8) {
@@ -240,7 +239,7 @@ int reconstruct_bwd_recompute_typed(const T* L, const T* A, const T* D, const T*
     return packed_bwd_typed<T, false>(L, A, D, p0, fd, n0, nullptr, nullptr, g, gL, gA, gD, B, N, st, anchor);
   return with_scan_plan(B, N - 3, [&]<int W, int K>() {
     return launch_chunks(B, 64 * W, [&](int64_t off, unsigned n) {
-      hipLaunchKernelGGL((reconstruct_backward_recompute_kernel<T, W, K, kScanPad>), dim3(n), dim3(64 * W), 0, st,
+      hipLaunchKernelGGL((reconstruct_backward_recompute_kernel<T, W, K>), dim3(n), dim3(64 * W), 0, st,
                          L + off * (N - 1), A + off * (N - 2), D + off * (N - 3), p0, fd, n0, g + off * N * 3,
                          gL + off * (N - 1), gA + off * (N - 2), gD + off * (N - 3), N,
                          anchor != nullptr ? anchor + off * 6 : nullptr);
@@ -459,7 +458,7 @@ int long_bwd_typed(const T* L, const T* A, const T* D, const T* p0, const T* fd,
                      dim3(kLongThreads), 0, st, state, work, B, segs);
   if (hipGetLastError() != hipSuccess) return CUFK_ERR_LAUNCH;
   return with_scan_plan(B * segs, S, [&]<int W, int K>() {
-    hipLaunchKernelGGL((long_backward_segments_kernel<T, W, K, kScanPad>), dim3(static_cast<unsigned>(B * segs)),
+    hipLaunchKernelGGL((long_backward_segments_kernel<T, W, K>), dim3(static_cast<unsigned>(B * segs)),
                        dim3(64 * W), 0, st, L, A, D, p0, fd, n0, xyz, local, flags, g, gL, gA, gD, state, work, N,
                        S, segs, anchor);
     return hipGetLastError() == hipSuccess ? CUFK_OK : CUFK_ERR_LAUNCH;

@@ -271,7 +271,7 @@ static __global__ __launch_bounds__(kLongThreads) void long_backward_carry_kerne
   }
 }
 
-template <typename T, int W, int K, int Pad>
+template <typename T, int W, int K>
 __global__ __launch_bounds__(64 * W) void long_backward_segments_kernel(
     const T* __restrict__ lengths, const T* __restrict__ angles, const T* __restrict__ dihedrals,
     const T* __restrict__ p0, const T* __restrict__ first_direction, const T* __restrict__ initial_normal,
@@ -280,7 +280,7 @@ __global__ __launch_bounds__(64 * W) void long_backward_segments_kernel(
     T* __restrict__ grad_dihedrals, const double* __restrict__ state, const double* __restrict__ work, int points,
     int seg_steps, int segments, double* __restrict__ anchor = nullptr) {
   using R = compute_t<T>;
-  using Lay = Layout<W, K, Pad>;
+  using Lay = Layout<W, K>;
   constexpr int kA = 3 * Lay::kStepRow > Lay::kPointRow ? 3 * Lay::kStepRow : Lay::kPointRow;
   __shared__ __align__(16) R pstage[kA];
   __shared__ __align__(16) R gstage[Lay::kPointRow];

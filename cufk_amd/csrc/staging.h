@@ -1,17 +1,13 @@
 // LDS staging of chain rows.
 //
 // Global rows are streamed with 16-byte vector accesses (coalesced across the workgroup) into
-// LDS layouts in which every lane's K steps (or K points) are contiguous, padded by Pad words
+// LDS layouts in which every lane's K steps (or K points) are contiguous, padded by one word
 // per lane:
-//   step layout:  step s        -> slot s + Pad*(s/K)              (lane stride K+Pad)
-//   point layout: flat xyz e>=9 -> slot 12 + e' + Pad*(e'/(3K))    (e' = e-9, lane stride 3K+Pad)
+//   step layout:  step s        -> slot s + s/K              (lane stride K+1)
+//   point layout: flat xyz e>=9 -> slot 12 + e' + e'/(3K)    (e' = e-9, lane stride 3K+1)
 //                 e < 9 (points 0..2) -> slot e
-// Lane t owns steps [tK, tK+K) and points [3+tK, 3+tK+K).
-//   Pad = 4 (K a multiple of 4): lane runs are 16-byte aligned and the strides are 4 mod 32
-//     words, so ds_read_b128 / ds_write_b128 by the lanes hit disjoint banks.
-//   Pad = 1: odd strides, so one 32-bit access per lane hits 64 distinct banks; every access
-//     is a 32-bit one and the layout is 3/4 the size of Pad = 4 at K = 8 (more workgroups per
-//     CU where LDS bounds occupancy).
+// Lane t owns steps [tK, tK+K) and points [3+tK, 3+tK+K).  The strides are odd, so one 32-bit access
+// per lane hits 64 distinct banks.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -58,24 +54,22 @@ template <bool Stream> __device__ __forceinline__ void global_store(f64x2u* p, f
     *p = v;
 }
 
-template <int W, int K, int Pad = 4> struct Layout {
+template <int W, int K> struct Layout {
   static_assert(K % 4 == 0, "lane segments must be whole 16-byte groups");
-  static_assert(Pad == 4 || Pad == 1, "padding is 4 words (vector LDS access) or 1 word");
   static constexpr int kWaves = W;
   static constexpr int kItems = K;
-  static constexpr int kPad = Pad;
+  static constexpr int kPad = 1;
   static constexpr int kLanes = 64 * W;
   static constexpr int kCap = kLanes * K;  // steps per chain
-  static constexpr bool kVec = Pad == 4;    // lane runs 16-byte aligned
-  static constexpr int kStepStride = K + Pad;
+  static constexpr int kStepStride = K + kPad;
   static constexpr int kStepRow = kLanes * kStepStride;
-  static constexpr int kPointStride = 3 * K + Pad;
+  static constexpr int kPointStride = 3 * K + kPad;
   static constexpr int kPointRow = 12 + kLanes * kPointStride;
-  __device__ __forceinline__ static int step_slot(int s) { return s + Pad * (s / K); }
+  __device__ __forceinline__ static int step_slot(int s) { return s + kPad * (s / K); }
   __device__ __forceinline__ static int point_slot(int e) {
     if (e < 9) return e;
     const int t = e - 9;
-    return 12 + t + Pad * (t / (3 * K));
+    return 12 + t + kPad * (t / (3 * K));
   }
   __device__ __forceinline__ static int lane_step_base(int tid) { return tid * kStepStride; }
   __device__ __forceinline__ static int lane_point_base(int tid) { return 12 + tid * kPointStride; }
@@ -201,26 +195,19 @@ __device__ __forceinline__ void store_windows(T* __restrict__ dst, const compute
   if (e < n) global_store<Stream>(dst + e, narrow<T>(src[Map::slot(x0 + e)]));
 }
 
-// A 16-byte group of consecutive LDS slots: one vector read when the layout keeps lane runs
-// 16-byte aligned, element reads otherwise.
-template <typename Lay, typename V, typename S> __device__ __forceinline__ V lds_vec(const S* p) {
-  if constexpr (Lay::kVec) {
-    return *reinterpret_cast<const V*>(p);
-  } else {
-    V v;
+// A 16-byte group of consecutive LDS slots.
+template <typename V, typename S> __device__ __forceinline__ V lds_vec(const S* p) {
+  V v;
 #pragma unroll
-    for (int e = 0; e < static_cast<int>(sizeof(V) / sizeof(S)); ++e) v[e] = p[e];
-    return v;
-  }
+  for (int e = 0; e < static_cast<int>(sizeof(V) / sizeof(S)); ++e) v[e] = p[e];
+  return v;
 }
 
 // One thread's share of NR rows moved into LDS, in two phases: fetch() issues the thread's
 // global loads of src[r][first, first + n) into registers; commit() writes them to
 // dst[r][Map::slot(first + e)] and returns whether any element of a row in RangeRows (bit r
 // for row r) lies beyond the polynomial range of sin_cos_wide.  MaxN bounds n at compile time.
-// A 16-byte group never straddles a lane segment, so its elements land in consecutive slots;
-// Vec writes it with one vector LDS store (slots 16-byte aligned), otherwise element by
-// element.
+// A 16-byte group never straddles a lane segment, so its elements land in consecutive slots.
 template <int NR, int MaxN, int Lanes, typename T, typename Map, bool Half = sizeof(T) == 2>
 struct RowFetch {  // float, double
   using R = compute_t<T>;
@@ -249,7 +236,7 @@ struct RowFetch {  // float, double
     }
   }
 
-  template <bool Vec, unsigned RangeRows>
+  template <unsigned RangeRows>
   __device__ __forceinline__ bool commit(R* const (&dst)[NR], int tid) const {
     bool wide = false;
 #pragma unroll
@@ -259,12 +246,8 @@ struct RowFetch {  // float, double
 #pragma unroll
         for (int r = 0; r < NR; ++r) {
           R* const d = dst[r] + Map::slot(first + E * g);
-          if constexpr (Vec) {
-            *reinterpret_cast<typename Unit<T>::Local*>(d) = buf[r][j];
-          } else {
 #pragma unroll
-            for (int e = 0; e < E; ++e) d[e] = buf[r][j][e];
-          }
+          for (int e = 0; e < E; ++e) d[e] = buf[r][j][e];
           if ((RangeRows >> r) & 1u) {
 #pragma unroll
             for (int e = 0; e < E; ++e) wide = wide || beyond_wide_reduce(buf[r][j][e]);
@@ -321,7 +304,7 @@ template <int NR, int MaxN, int Lanes, typename T, typename Map> struct RowFetch
     }
   }
 
-  template <bool Vec, unsigned RangeRows>
+  template <unsigned RangeRows>
   __device__ __forceinline__ bool commit(R* const (&dst)[NR], int tid) const {
     // Largest magnitude patterns staged from the rows in RangeRows, two lanes of 16 bits: the
     // windows' dwords are masked and maximised whole (v_pk_max_u16).
@@ -365,18 +348,18 @@ template <int NR, int MaxN, int Lanes, typename T, typename Map> struct RowFetch
 // workgroup pays one memory latency per staging phase, not one per group.  Returns whether
 // any element this thread staged from a row in RangeRows lies beyond the polynomial range of
 // sin_cos_wide (RowFetch).
-template <int NR, int MaxN, int Lanes, bool Vec, typename Map, unsigned RangeRows = 0, typename T>
+template <int NR, int MaxN, int Lanes, typename Map, unsigned RangeRows = 0, typename T>
 __device__ __forceinline__ bool stage_rows(compute_t<T>* const (&dst)[NR], const T* const (&src)[NR], int first, int n,
                                            int tid) {
   RowFetch<NR, MaxN, Lanes, T, Map> rows;
   rows.fetch(src, first, n, tid);
-  return rows.template commit<Vec, RangeRows>(dst, tid);
+  return rows.template commit<RangeRows>(dst, tid);
 }
 
 // NR step rows (n <= kCap elements each) into step layouts; see stage_rows for RangeRows.
 template <typename Lay, int NR, unsigned RangeRows = 0, typename T>
 __device__ __forceinline__ bool load_step_rows(compute_t<T>* const (&dst)[NR], const T* const (&src)[NR], int n, int tid) {
-  return stage_rows<NR, Lay::kCap, Lay::kLanes, Lay::kVec, StepRowMap<Lay>, RangeRows, T>(dst, src, 0, n, tid);
+  return stage_rows<NR, Lay::kCap, Lay::kLanes, StepRowMap<Lay>, RangeRows, T>(dst, src, 0, n, tid);
 }
 
 // NR (points, 3) rows into point layouts.
@@ -387,7 +370,7 @@ __device__ __forceinline__ void load_point_rows(compute_t<T>* const (&dst)[NR], 
 #pragma unroll
     for (int r = 0; r < NR; ++r) dst[r][tid] = widen(src[r][tid]);
   }
-  stage_rows<NR, 3 * Lay::kCap, Lay::kLanes, Lay::kVec, PointRowMap<Lay>, 0u, T>(dst, src, 9, 3 * points - 9, tid);
+  stage_rows<NR, 3 * Lay::kCap, Lay::kLanes, PointRowMap<Lay>, 0u, T>(dst, src, 9, 3 * points - 9, tid);
 }
 
 // One lane's run of n <= N consecutive elements between global memory and registers, in
@@ -439,45 +422,6 @@ __device__ __forceinline__ void store_run(T* __restrict__ dst, int n, const comp
     if (j < n) global_store<Stream>(dst + j, narrow<T>(src[j]));
 }
 
-// dst[s] = src[step_slot(s)] for s in [0, n).
-template <typename Lay, typename T>
-__device__ __forceinline__ void store_step_row(T* __restrict__ dst, const compute_t<T>* __restrict__ src, int n, int tid) {
-  if constexpr (std::is_same_v<T, float>) {
-    const int groups = n >> 2;
-    for (int g = tid; g < groups; g += Lay::kLanes)
-      *reinterpret_cast<f32x4u*>(dst + 4 * g) = lds_vec<Lay, f32x4>(src + Lay::step_slot(4 * g));
-    for (int s = 4 * groups + tid; s < n; s += Lay::kLanes) dst[s] = src[Lay::step_slot(s)];
-  } else if constexpr (std::is_same_v<T, double>) {
-    const int groups = n >> 1;
-    for (int g = tid; g < groups; g += Lay::kLanes)
-      *reinterpret_cast<f64x2u*>(dst + 2 * g) = lds_vec<Lay, f64x2>(src + Lay::step_slot(2 * g));
-    if ((n & 1) && tid == 0) dst[n - 1] = src[Lay::step_slot(n - 1)];
-  } else {
-    for (int s = tid; s < n; s += Lay::kLanes) dst[s] = narrow<T>(src[Lay::step_slot(s)]);
-  }
-}
-
-// dst[e] = src[point_slot(e)] for e in [0, 3*points); without `head`, points 0..2 are left alone.
-template <typename Lay, bool Stream = false, typename T>
-__device__ __forceinline__ void store_point_row(T* __restrict__ dst, const compute_t<T>* __restrict__ src, int points,
-                                                int tid, bool head = true) {
-  const int n = 3 * points - 9;
-  if (head && tid < 9) global_store<Stream>(dst + tid, narrow<T>(src[tid]));
-  if constexpr (std::is_same_v<T, float>) {
-    const int groups = n >> 2;
-    for (int g = tid; g < groups; g += Lay::kLanes)
-      global_store<Stream>(reinterpret_cast<f32x4u*>(dst + 9 + 4 * g), f32x4u(lds_vec<Lay, f32x4>(src + Lay::point_slot(9 + 4 * g))));
-    for (int e = 4 * groups + tid; e < n; e += Lay::kLanes) global_store<Stream>(dst + 9 + e, src[Lay::point_slot(9 + e)]);
-  } else if constexpr (std::is_same_v<T, double>) {
-    const int groups = n >> 1;
-    for (int g = tid; g < groups; g += Lay::kLanes)
-      global_store<Stream>(reinterpret_cast<f64x2u*>(dst + 9 + 2 * g), f64x2u(lds_vec<Lay, f64x2>(src + Lay::point_slot(9 + 2 * g))));
-    if ((n & 1) && tid == 0) global_store<Stream>(dst + 9 + n - 1, src[Lay::point_slot(9 + n - 1)]);
-  } else {
-    store_windows<Lay::kLanes, PointRowMap<Lay>, Stream>(dst + 9, src, 9, n, tid);
-  }
-}
-
 // Three step-indexed gradient rows written interleaved into the point layout: the outputs of
 // step s (lane t, item i) occupy slots lane_point_base(t) + 3i + {0,1,2}, i.e. exactly the
 // upstream-gradient slots of point s+3, which the owning lane has consumed by then.
@@ -489,9 +433,9 @@ __device__ __forceinline__ void store_interleaved_rows(T* __restrict__ a, T* __r
     const int groups = steps >> 2;  // 4 steps never straddle a lane (K % 4 == 0)
     for (int g = tid; g < groups; g += Lay::kLanes) {
       const float* p = src + Lay::point_slot(9 + 12 * g);
-      const f32x4 v0 = lds_vec<Lay, f32x4>(p);
-      const f32x4 v1 = lds_vec<Lay, f32x4>(p + 4);
-      const f32x4 v2 = lds_vec<Lay, f32x4>(p + 8);
+      const f32x4 v0 = lds_vec<f32x4>(p);
+      const f32x4 v1 = lds_vec<f32x4>(p + 4);
+      const f32x4 v2 = lds_vec<f32x4>(p + 8);
       global_store<true>(reinterpret_cast<f32x4u*>(a + 4 * g), f32x4u{v0.x, v0.w, v1.z, v2.y});
       global_store<true>(reinterpret_cast<f32x4u*>(b + 4 * g), f32x4u{v0.y, v1.x, v1.w, v2.z});
       global_store<true>(reinterpret_cast<f32x4u*>(c + 4 * g), f32x4u{v0.z, v1.y, v2.x, v2.w});
