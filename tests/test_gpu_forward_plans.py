@@ -60,7 +60,7 @@ def test_plan_edges_small_batches(device, dtype, steps):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16", "float16"])
 @pytest.mark.parametrize("batch,steps", [(2048, 300), (2049, 300), (2049, 511), (2048, 520), (2049, 520), (2049, 765),
                                          (2049, 768), (1024, 800), (1025, 801), (2049, 1023)])
 def test_plan_edges_large_batches(device, dtype, batch, steps):

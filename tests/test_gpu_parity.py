@@ -659,8 +659,8 @@ def _abi_fused():
     return lib
 
 
-@pytest.mark.parametrize("dtype", [torch.float32, torch.float64, torch.bfloat16])
-@pytest.mark.parametrize("B,N", [(40, 300), (9, 2049), (4100, 64)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,N", [(40, 300), (9, 2049), (4100, 64), (2049, 300), (2049, 700), (1100, 900)])
 def test_fused_forwards_store_the_flagged_forwards_positions(device, dtype, B, N):
     """The fused-loss forwards (squared distance, superposed) write xyz and the regularity flags
     as cufk_reconstruct_fwd_flagged does: bit for bit where that entry point runs one chain per
@@ -679,7 +679,7 @@ def test_fused_forwards_store_the_flagged_forwards_positions(device, dtype, B, N
     target = (xyz.double() + 0.3 * torch.randn(B, N, 3, device=device, dtype=torch.float64)).to(dtype)
     packed = B >= 4096 and N - 3 <= 128
     scale = max(1.0, float(xyz.double().abs().max()))
-    tol = {torch.float32: 2e-6, torch.float64: 1e-12, torch.bfloat16: 2.0**-7}[dtype] * scale
+    tol = {torch.float32: 2e-6, torch.float64: 1e-12, torch.bfloat16: 2.0**-7, torch.float16: 2.0**-10}[dtype] * scale
 
     def same(got, got_reg, what):
         if packed:
@@ -703,7 +703,7 @@ def test_fused_forwards_store_the_flagged_forwards_positions(device, dtype, B, N
                                                      p(x2), p(r2), p(loss), p(rec), B, N, st)
         assert rc == 0, what
         same(x2, r2, what)
-    if dtype == torch.bfloat16 and lib.cufk_reconstruct_shadow_floats(B, N) > 0:
+    if dtype in (torch.bfloat16, torch.float16) and lib.cufk_reconstruct_shadow_floats(B, N) > 0:
         x3 = torch.empty_like(xyz)
         pos = torch.empty(B, N, 3, device=device, dtype=torch.float32)
         r3 = torch.full((B,), 7, device=device, dtype=torch.uint8)

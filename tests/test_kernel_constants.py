@@ -128,3 +128,38 @@ def test_a_wrong_table_entry_is_caught(entry):
     x = _angles()
     s, _ = _sin_cos(x, k_round, inv_step, step, s1, c2, bad)
     assert np.abs(s - np.sin(x.astype(np.float64))).max() > 1e-11
+
+
+def _serial_rows(L, s, c, S, C, rows, dtype):
+    """A lane's serial scan (run_scan): the third row of every prefix rotation tracked, or (rows = 2) the
+    cross product of the other two; the last rotation and translation."""
+    L, s, c, S, C = (v.astype(dtype) for v in (L, s, c, S, C))
+    m = [[-c[0], -s[0], np.zeros_like(c[0])], [s[0] * C[0], -c[0] * C[0], -S[0]], [s[0] * S[0], -c[0] * S[0], C[0]]]
+    v = [L[0] * row[0] for row in m]
+    for i in range(1, len(L)):
+        for r in range(rows):
+            a1, a2 = C[i] * m[r][1] + S[i] * m[r][2], C[i] * m[r][2] - S[i] * m[r][1]
+            m[r] = [s[i] * a1 - c[i] * m[r][0], -s[i] * m[r][0] - c[i] * a1, a2]
+            v[r] = v[r] + L[i] * m[r][0]
+        if rows == 2:
+            (a, b, d), (e, f, g) = m[:2]
+            m[2] = [b * g - d * f, d * e - a * g, a * f - b * e]
+            v[2] = v[2] + L[i] * m[2][0]
+    return np.array([*m[2], v[2]])
+
+
+@pytest.mark.parametrize("steps", [4, 8, 12])
+def test_third_row_from_the_other_two_loses_nothing(steps):
+    """Against extended precision over the bench's angles: the error of the third rotation row and of the
+    translation along it is the table's, whether the row is tracked or follows from the first two."""
+    rng = np.random.default_rng(3)
+    shape = (steps, 40_000)
+    A = rng.normal(2.05, 0.08, shape).astype(np.float32)
+    D = rng.uniform(-np.pi, np.pi, shape).astype(np.float32)
+    L = np.clip(rng.normal(0.145, 0.01, shape), 0.12, 0.17).astype(np.float32)
+    table = [*_sin_cos(A, *_constants()), *_sin_cos(D, *_constants())]
+    exact = [f(x.astype(np.longdouble)) for x in (A, D) for f in (np.sin, np.cos)]
+    want = _serial_rows(L, *exact, 3, np.longdouble)
+    err = [np.sqrt(np.square((_serial_rows(L, *table, rows, np.float64) - want).astype(np.float64)).mean(1)) for rows in (2, 3)]
+    print(f"{steps} steps: rms errors of the row and the translation, two rows {err[0]}, three {err[1]}")
+    assert (err[0] <= 1.01 * err[1]).all()
