@@ -107,15 +107,15 @@ ELEM_BYTES = {"float32": 4, "float64": 8, "float16": 2, "bfloat16": 2}
 # backward launches: profiles/counters_and_traffic_bench_regime.md.  A config without an entry
 # reports traffic and roofline_valu as null.
 MEASURED_TRAFFIC = {
-    "c1": 24429892, "c2": 510976820, "c2_far": 511569622, "c2_mixed": 511340596, "c3": 380682861,
-    "c4_bf16": 827142795, "long": 914240077, "loss": 613084106, "rmsd": 616138701, "torsion_loss": 458950537,
-    "short": 500206727,
+    "c1": 24460117, "c2": 509416723, "c2_far": 510663297, "c2_mixed": 510265526, "c3": 380691071,
+    "c4_bf16": 827656085, "long": 914950353, "loss": 611538543, "rmsd": 615308795, "torsion_loss": 458941146,
+    "short": 502829489,
 }
 MEASURED_VALU = {  # (forward, backward) per launch
-    "c1": (1796096, 1122816), "c2": (20185088, 14049280), "c2_far": (20185088, 49795072),
-    "c2_mixed": (20184064, 22985728), "c3": (10616832, 11608064), "c4_bf16": (42958848, 30072832),
-    "long": (22353856, 22759616), "loss": (22122496, 14872576), "rmsd": (36209664, 18583002),
-    "torsion_loss": (12034048, 12230656), "short": (27754496, 23560192),
+    "c1": (1686528, 982528), "c2": (18718720, 12812288), "c2_far": (18718720, 49090560),
+    "c2_mixed": (18717696, 21881856), "c3": (9486336, 11608064), "c4_bf16": (39796736, 26517504),
+    "long": (21227392, 23533760), "loss": (21073920, 13852672), "rmsd": (28685312, 17538539),
+    "torsion_loss": (10993664, 12230656), "short": (21643294, 23560192),
 }
 # VALU issue peak: 1024 SIMDs (256 CUs x 4) at 2.4 GHz, one wave64 instruction per 4 cycles each.
 VALU_PEAK_PER_S = 1024 * 2.4e9 / 4
