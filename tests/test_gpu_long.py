@@ -182,7 +182,7 @@ def test_long_position_adjoint_far_anchor_and_boundary_bonds(cufk, device):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_long_angles_beyond_the_polynomial_range(cufk, device, dtype):
-    """Angles with |x| > 65536 in non-head segments switch those segments to the library
+    """Angles with |x| > 65536 in non-head segments switch those segments to the checked
     sin/cos; float32 bars as above, bfloat16 2e-2 relative to the chain extent."""
     d = _inputs(3, 300, seed=12, anchors=True, dtype=dtype)
     d["dihedrals"][0, 150] += 2 * math.pi * 20000.0

@@ -1053,8 +1053,8 @@ def test_half_autograd_takes_the_float_positions(cufk, device):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_angles_beyond_the_polynomial_range(cufk, device, dtype):
-    """Angles with |x| > 65536 take the library sin/cos (the kernels switch the whole chain to
-    the checked loop).  Chain 0 is ordinary, chain 1 regular with one huge dihedral, chain 2
+    """Angles with |x| > 65536 take the checked sin/cos (the forwards' exact reduction, the backwards'
+    library routine; a wave or a chain switches as a whole).  Chain 0 is ordinary, chain 1 regular with one huge dihedral, chain 2
     irregular (negative bond) with a huge dihedral and a huge bond angle, chain 3 a huge
     angle near a lane boundary.  Forward, the one-launch backward and the exact backward
     against the oracle on the same (dtype-rounded) inputs; fp32 tolerances as above, bf16
